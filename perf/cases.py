@@ -93,10 +93,11 @@ def draw(rng):
     if kind == "conv":
         weights = rng.choice(["binary", "ternary", "f32", "tbn"])
         c = _log_int(rng, 3 if weights == "f32" else 16, 512)
-        m = _log_int(rng, 16, 512)
         hw = _log_int(rng, 7, 112)
+        # the conv layout's patches: stride 2 up to 3x3 and from 33 output channels
         k = rng.choice([1, 3, 3, 5])
         stride = rng.choice([1, 1, 2]) if k < 5 else 1
+        m = _log_int(rng, 16 if stride == 1 else 33, 512)
         n = _log_int(rng, 1, 64)
         out = (hw + 2 * (k // 2) - k) // stride + 1
         while n > 1 and 2.0 * n * m * c * k * k * out * out > 16e9:
