@@ -390,6 +390,50 @@ def test_gemm_f32_rows_and_split_k(dev, orc):
             assert np.array_equal(host(few), host(out)[3:5])
 
 
+# every tile of the fp32 kernel (64 x 64, 32 x 32, 16 x 16 with short and long
+# chunks), one past and one short of a tile, K of one value, around an
+# instruction's 4 and a step's 16 values and around a chunk
+@pytest.mark.parametrize("M,K,N", [(1500, 130, 1300), (1409, 63, 1409), (500, 65, 530), (513, 64, 513), (300, 127, 520),
+                                   (290, 129, 470), (1, 1, 65), (15, 3, 66), (17, 4, 4096), (16, 255, 80), (33, 257, 79),
+                                   (2, 4096, 67), (3, 17, 1001)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+def test_gemm_f32_dense_tiles(dev, M, K, N, ta, tb):
+    """fp32 GEMM against float64; a row of the full call has the bits of the
+    same row in a call of two rows (another tile), infinities and NaN reach
+    exactly their row, and nothing is written past the output."""
+    rng = np.random.default_rng(M + K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    c1 = rng.standard_normal(N).astype(np.float32)
+    dB = to_dev(np.ascontiguousarray(B.T) if tb else B)
+
+    def gemm(rows):
+        m = rows.shape[0]
+        out = torch.full((m * N + 64,), float("nan"), device=dev)
+        a = to_dev(np.ascontiguousarray(rows.T) if ta else np.ascontiguousarray(rows))
+        tbn_hip.call("tbn_hip_gemm_f32", P(a), P(dB), P(to_dev(c1)), 1, m, K, N, 0.5, 2.0, int(ta), int(tb), 0,
+                     P(out), None)
+        full = host(out)
+        assert np.isnan(full[m * N:]).all(), "written past the output"
+        return full[:m * N].reshape(m, N)
+
+    y = gemm(A)
+    ref = 0.5 * (A.astype(np.float64) @ B.astype(np.float64)) + 2.0 * c1
+    # K rounded sums and the two epilogue steps, each at most half an ulp of a
+    # partial sum of at most sum |a*b| + |c|
+    bound = (K + 4) * 2.0 ** -24 * (0.5 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)) + 2 * np.abs(c1))
+    assert (np.abs(y - ref) <= bound).all()
+    pick = np.array([M - 1, M // 2])
+    assert np.array_equal(gemm(A[pick]).view(np.uint32), y[pick].view(np.uint32))
+    bad = A.copy()
+    bad[M // 2, K - 1] = np.inf
+    bad[M - 1, 0] = np.nan
+    z = gemm(bad)
+    other = np.setdiff1d(np.arange(M), [M // 2, M - 1])
+    assert np.array_equal(z[other].view(np.uint32), y[other].view(np.uint32))
+    assert np.isnan(z[M - 1]).all() and (M // 2 == M - 1 or np.isinf(z[M // 2]).all())
+
+
 def test_gemm_error_codes(dev):
     packed = empty(64, torch.uint8)
     A = empty((4, 64), torch.float32)
