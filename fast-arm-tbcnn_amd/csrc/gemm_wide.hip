@@ -136,7 +136,7 @@ gemm_wide_kernel(tbn_hip::WideGemmArgs p, int tiles_r, int tiles_c, int steps_pe
     // A staging: thread -> row ar, EPT consecutive k from ag * EPT
     const int ar = tid / Cfg::TPR, ag = tid % Cfg::TPR;
     const float* a_base = p.A + static_cast<int64_t>(r0) * p.lda;
-    const uint64_t a_bytes = static_cast<uint64_t>(p.M - r0) * p.lda * 4;
+    const uint64_t a_bytes = (static_cast<uint64_t>(p.M - 1 - r0) * p.lda + p.K) * 4;
     const int a_voff = (ar * static_cast<int>(p.lda) + ag * Cfg::EPT) * 4;
     // W: lane's columns c0 + wc*WC + j*32 + lane%32
     const uint8_t* b_base = p.packed + static_cast<int64_t>(c0) * p.col_bytes;
@@ -472,8 +472,9 @@ gemm_mid_kernel(tbn_hip::WideGemmArgs p, int tiles_r, int tiles_c, int steps_per
     const int r0 = tr * Cfg::BR;
     const int c0 = tc * Cfg::BC;
     const int all_steps = (p.K + KS - 1) / KS;
-    // a K group's steps: the host gives each group the same count
-    const int per_group = (SPLIT ? steps_per_split : all_steps) / Cfg::KG;
+    // a K group's steps: every group the same count (the barriers are shared);
+    // a step past K reads zeros
+    const int per_group = ((SPLIT ? steps_per_split : all_steps) + Cfg::KG - 1) / Cfg::KG;
     const int s0 = (SPLIT ? split * steps_per_split : 0) + kgrp * per_group;
     const int ns = SPLIT ? min(per_group, all_steps - s0) : per_group;
 
@@ -498,7 +499,7 @@ gemm_mid_kernel(tbn_hip::WideGemmArgs p, int tiles_r, int tiles_c, int steps_per
     // A staging: thread -> row ar, EPT consecutive k from ag * EPT
     const int ar = tid / Cfg::TPR, ag = tid % Cfg::TPR;
     const float* a_base = p.A + static_cast<int64_t>(r0) * p.lda;
-    const uint64_t a_bytes = static_cast<uint64_t>(p.M - r0) * p.lda * 4;
+    const uint64_t a_bytes = (static_cast<uint64_t>(p.M - 1 - r0) * p.lda + p.K) * 4;
     const int a_voff = (ar * static_cast<int>(p.lda) + ag * Cfg::EPT) * 4;
     // W: lane's columns c0 + wc*WC + j*32 + lane%32
     const uint8_t* b_base = p.packed + static_cast<int64_t>(c0) * p.col_bytes;
@@ -887,19 +888,21 @@ gemm_mid_kernel(tbn_hip::WideGemmArgs p, int tiles_r, int tiles_c, int steps_per
     }
 }
 
-// Tile and K-split choice.  Shapes whose 128 x 512 tiles fill the chip (>= 128
-// blocks of 8 waves) take them whole.  Others with an even number of K steps
-// whose 32 x 128 tiles number at least 256 take those, in two K groups (one
-// block of 8 waves per CU, no partial sums through memory; config 2, 1024^3:
-// 10.2 us kernel time against 15.2 for the 64 x 128 tile split 4 ways).  The
-// rest take the 64 x 128 tile with K split over up to 8 blocks per tile,
-// aiming at 512 blocks (two per CU), each split keeping at least 4 K steps
-// (config 3, 256 x 4096^2 ternary: 4 splits 36.6 us, 2 splits 42.7, 8 splits
-// 40.4; the 128 x 512 and 128 x 256 tiles with any split were slower).  The
-// choice reads only M, N and K, so a GEMM's result does not depend on
-// anything else.  TBN_TUNE_GEMM_TILE / TBN_TUNE_GEMM_SPLITS force either.
+// Tile choice.  Shapes whose 128 x 512 tiles fill the chip (>= 128 blocks of 8
+// waves) take them.  Others with at least 160 tiles of 32 x 128 and a K of 65
+// to 1100 take those, in two K groups: their staging splits A once per 64 k
+// for four waves and has little to add at the end (2000 x 600 x 1000 13.6 us
+// against 15.7 for the best of gemm_waves.hip, 1000 x 1200 x 1000 13.9
+// against 13.5, 777 x 1333 x 1001 14.0 against 14.3, 300 x 2000 x 2000 17.7 against 16.1).  The
+// rest splits K over the waves of a block (gemm_waves.hip); beyond 256 tiles of 32 x 128
+// with K of 64 or less the 64 x 64 tile of gemm.hip stays (4096 x 64 x 4096
+// 18 us against 82).  The choice reads only M, N and K, so a GEMM's result
+// does not depend on anything else.  TBN_TUNE_GEMM_TILE /
+// TBN_TUNE_GEMM_SPLITS force a tile of this file (the 64 x 128 tile with K
+// split over blocks through memory is reached only that way).
 struct WidePlan {
-    int cfg = 0;      // 0 Wide, 1 WideSmall, 2 WideMid
+    int cfg = 0;      // 0 Wide, 1 WideSmall, 2 WideMid, 3 gemm_waves.hip, 4 none of them
+    int waves = 0;    // cfg 3: the variant
     int tiles_r = 0, tiles_c = 0, steps = 0, splits = 1, per = 0;
     int xcd_cols = 1;  // mid-size tiles: XCD grid columns (gemm_mid_kernel's tile order)
     int64_t blocks() const { return static_cast<int64_t>(tiles_r) * tiles_c * splits; }
@@ -942,21 +945,20 @@ WidePlan plan_for(int cfg, int M, int N, int K, bool ternary) {
     return w;
 }
 
-// WideMid needs an even step count (its two K groups take equal halves).
-bool mid_ok(int K) { return tbn_hip::ceil_div(K, WideMid::KS) % 2 == 0; }
-
 WidePlan choose_plan(int M, int N, int K, bool ternary) {
     const int forced = tbn_hip::tuning(TBN_TUNE_GEMM_TILE);
     if (forced == 0) return plan_for<Wide>(0, M, N, K, ternary);
     if (forced == 1) return plan_for<WideSmall>(1, M, N, K, ternary);
-    if (forced == 2 && mid_ok(K)) return plan_for<WideMid>(2, M, N, K, ternary);
+    if (forced == 2) return plan_for<WideMid>(2, M, N, K, ternary);
     const WidePlan big = plan_for<Wide>(0, M, N, K, ternary);
     if (big.blocks() >= 128) return big;
-    if (forced != 1 && mid_ok(K)) {
-        const WidePlan mid = plan_for<WideMid>(2, M, N, K, ternary);
-        if (mid.blocks() >= 256 && mid.steps >= 4) return mid;
-    }
-    return plan_for<WideSmall>(1, M, N, K, ternary);
+    if (tbn_hip::tuning(TBN_TUNE_GEMM_SPLITS) >= 1) return plan_for<WideSmall>(1, M, N, K, ternary);
+    const WidePlan mid = plan_for<WideMid>(2, M, N, K, ternary);
+    if (mid.blocks() >= 160 && mid.steps >= 2 && K < 1100) return mid;
+    WidePlan w;
+    w.cfg = mid.blocks() > 256 && K <= 64 ? 4 : 3;
+    w.waves = tbn_hip::gemm_waves_plan(M, N, K);
+    return w;
 }
 
 // Kernel variants: the large tile on gemm_wide_kernel, the mid-size (DEEP)
@@ -998,19 +1000,21 @@ namespace tbn_hip {
 
 bool gemm_wide_fits(const WideGemmArgs& a, bool ternary) {
     const WidePlan w = choose_plan(a.M, a.N, a.K, ternary);
-    const int waves = w.cfg == 1 ? 4 : 8;
     const int bc = w.cfg == 0 ? 512 : 128;
-    // shapes that give at least half the chip one wave per SIMD
-    return a.K >= 64 && w.blocks() * waves >= 512 && a.M >= 64 && a.N >= 128 && a.lda % 4 == 0 &&
-           reinterpret_cast<uintptr_t>(a.A) % 16 == 0 && a.col_bytes % 16 == 0 &&
-           reinterpret_cast<uintptr_t>(a.packed) % 16 == 0 && a.lda <= (1 << 22) &&
-           static_cast<int64_t>(bc) * a.col_bytes < (1LL << 31) && (ternary || a.col_bytes % 16 == 0) &&
+    if (w.cfg == 4 || a.K < 1 || reinterpret_cast<uintptr_t>(a.packed) % 4 || a.lda > (1 << 22) ||
+        static_cast<int64_t>(bc) * a.col_bytes >= (1LL << 31))
+        return false;
+    if (w.cfg == 3) return true;
+    // a forced tile: shapes that give at least half the chip one wave per SIMD
+    const int waves = w.cfg == 1 ? 4 : 8;
+    return w.blocks() * waves >= 512 && a.K >= 64 &&
            static_cast<int64_t>(w.tiles_r) * w.tiles_c <= kWorkspaceCounters &&
            (w.splits == 1 || static_cast<int64_t>(a.M + 128) * a.N * 4 < (1LL << 31));
 }
 
 std::string gemm_wide_kernel_name(const WideGemmArgs& a, bool ternary) {
     const WidePlan w = choose_plan(a.M, a.N, a.K, ternary);
+    if (w.cfg == 3) return gemm_waves_kernel_name(w.waves, ternary);
     const char* cfg = w.cfg == 0   ? "WideCfg<128, 512, 128, 64, 64, false, 1>"
                       : w.cfg == 1 ? "WideCfg<64, 128, 32, 64, 64, true, 1>"
                                    : "WideCfg<32, 128, 32, 32, 64, true, 2>";
@@ -1021,6 +1025,7 @@ std::string gemm_wide_kernel_name(const WideGemmArgs& a, bool ternary) {
 
 int gemm_wide(const WideGemmArgs& a, bool ternary, hipStream_t stream) {
     const WidePlan w = choose_plan(a.M, a.N, a.K, ternary);
+    if (w.cfg == 3) return gemm_waves(a, ternary, w.waves, stream);
     const char* what = ternary ? "gemm_f32_ternary (wide)" : "gemm_f32_binary (wide)";
     void* part = nullptr;
     int* counters = nullptr;

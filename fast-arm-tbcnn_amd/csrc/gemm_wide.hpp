@@ -26,16 +26,21 @@ struct WideGemmArgs {
     int flags;
 };
 
-// True when the wide kernel takes this GEMM: enough tiles (with K splits) to
-// fill the chip, 16-byte aligned fp32 rows and 16-byte multiple packed columns.
-// `packed` holds BinaryMatrix columns, or 2-bit ternary columns when ternary.
+// True when one of the tiled kernels below takes this GEMM (dword-aligned
+// packed columns, byte offsets within a tile below 2^31).  `packed` holds
+// BinaryMatrix columns, or 2-bit ternary columns when ternary.
 bool gemm_wide_fits(const WideGemmArgs& a, bool ternary);
-// Runs it; shapes with few tiles split K over blocks, the last block of each
-// tile adding the splits in split order (stream workspace of splits * M * N
-// floats).
+// Runs it; a forced K split over blocks has the last block of each tile add
+// the splits in split order (stream workspace of splits * M * N floats).
 int gemm_wide(const WideGemmArgs& a, bool ternary, hipStream_t stream);
 // The kernel gemm_wide launches for this shape now (tuning controls
 // included), as a profiler names it.
 std::string gemm_wide_kernel_name(const WideGemmArgs& a, bool ternary);
+
+// K split over the waves of a block (gemm_waves.hip): a variant for a shape,
+// its kernel's name, and the launch.
+int gemm_waves_plan(int M, int N, int K);
+std::string gemm_waves_kernel_name(int plan, bool ternary);
+int gemm_waves(const WideGemmArgs& a, bool ternary, int plan, hipStream_t stream);
 
 }  // namespace tbn_hip

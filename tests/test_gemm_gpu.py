@@ -483,6 +483,15 @@ def make_wide_operands(rng, M, K, N, ternary):
     return A, scale, bias, packed, K_pad, N_pad, ref
 
 
+def gpu_unpack(packed, K, N, K_pad, ternary):
+    """The weights [K, N] as float64, decoded on the host from the packed columns."""
+    cols = host(packed).reshape(-1, K_pad // (4 if ternary else 8))[:N]
+    if ternary:
+        codes = (cols[:, :, None] >> (2 * np.arange(4))) & 3
+        return np.float64([-1, 0, 1, 0])[codes.reshape(N, K_pad)[:, :K]].T
+    return 1.0 - 2.0 * np.unpackbits(cols, axis=1, bitorder="little")[:, :K].T
+
+
 @pytest.mark.parametrize("tile,splits", sorted(WIDE_CASES))
 @pytest.mark.parametrize("ternary", [False, True], ids=["binary", "ternary"])
 def test_gemm_wide_every_tile_and_split(dev, orc, tile, splits, ternary):
@@ -531,6 +540,62 @@ def test_gemm_wide_leaves_memory_past_the_output_alone(dev, orc, tile, splits, t
     assert np.array_equal(out[:M, :N].view(np.uint32), plain.view(np.uint32))
     assert np.array_equal(out[M:].view(np.uint32), guard[M:]), "rows past M were written"
     assert np.array_equal(out[:, N:].view(np.uint32), guard[:, N:]), "columns past N were written"
+
+
+# each variant of the K-split-over-waves kernel, with ragged rows and columns,
+# fewer steps than waves, a K that ends inside a 32-step, and row strides that
+# are not a multiple of four floats
+WAVES_CASES = [("16, 1, 8", 1, 1, 67), ("16, 1, 8", 15, 33, 130), ("16, 1, 8", 17, 2829, 155), ("16, 1, 8", 64, 255, 90),
+               ("16, 2, 8", 24, 1031, 4095), ("16, 2, 8", 688, 735, 126), ("16, 2, 4", 291, 410, 383),
+               ("16, 2, 4", 600, 31, 420), ("16, 4, 8", 63, 1500, 3001), ("32, 2, 8", 130, 701, 2100),
+               ("32, 4, 8", 777, 1333, 1001), ("32, 4, 8", 300, 1130, 2000), ("32, 4, 4", 1100, 1129, 1025)]
+
+
+@pytest.mark.parametrize("ternary", [False, True], ids=["binary", "ternary"])
+@pytest.mark.parametrize("variant,M,K,N", WAVES_CASES)
+def test_gemm_waves_variants(dev, orc, variant, M, K, N, ternary):
+    """The variant runs, matches float64 within its rounding bound with and
+    without padded rows, an addend and either epilogue order, writes nothing outside
+    C, and carries infinities and NaN of a row to exactly that row."""
+    rng = np.random.default_rng(M * 7 + K + N + ternary)
+    A, scale, bias, packed, K_pad, N_pad, _ = make_wide_operands(rng, M, K, N, ternary)
+    kind = "ternary" if ternary else "binary"
+    assert gemm_kernel_name(ternary, M, N, K, K_pad, N_pad).startswith(f"gemm_waves_kernel<WavesCfg<{variant}>")
+    W = gpu_unpack(packed, K, N, K_pad, ternary)
+    ref = A.astype(np.float64) @ W
+    cin = rng.standard_normal((M, N)).astype(np.float32)
+    # every product is exact: K - 1 rounded additions and at most 4 epilogue steps
+    room = (K + 8) * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(W)) * np.abs(scale) * 1.5
+    room += 4 * 2.0 ** -23 * (np.abs(cin) + np.abs(bias) + 1)
+    for lda, ldc, flags, addend in [(K, N, 0, False), (K + 3, N + 5, tbn_hip.EPI_RELU, True),
+                                    (K + 1, N, tbn_hip.EPI_BIAS_THEN_SCALE, True)]:
+        wide = np.full((M, lda), np.nan, np.float32)
+        wide[:, :K] = A
+        dA = to_dev(np.concatenate([np.float32([np.nan]), wide.reshape(-1)]))  # rows start off a 16-byte boundary
+        out = torch.full(((M + 4) * ldc,), float("nan"), device=dev)
+        tbn_hip.call("tbn_hip_gemm_f32_quantized", int(ternary), dA.data_ptr() + 4, lda, M, N, K, P(packed), K_pad,
+                     N_pad, P(to_dev(scale)), 0.5, P(to_dev(bias)), P(to_dev(cin)) if addend else None, 0, 0.25, flags,
+                     P(out), ldc, None)
+        full = host(out)
+        y = full[:M * ldc].reshape(M, ldc)
+        want = (ref + bias) * (0.5 * scale) if flags & tbn_hip.EPI_BIAS_THEN_SCALE else ref * (0.5 * scale) + bias
+        want = want + (0.25 * cin if addend else 0.0)
+        if flags & tbn_hip.EPI_RELU:
+            want = np.maximum(want, 0.0)
+        assert (np.abs(y[:, :N] - want) <= room).all(), (lda, ldc, flags)
+        assert np.isnan(y[:, N:]).all() and np.isnan(full[M * ldc:]).all(), "written outside C"
+    bad = A.copy()
+    bad[M // 2, K - 1] = np.inf
+    bad[M - 1, K // 2] = np.nan
+    plain = host(run_gemm(kind, A, K, M, N, K, packed, K_pad, N_pad, scale))
+    z = host(run_gemm(kind, bad, K, M, N, K, packed, K_pad, N_pad, scale))
+    other = np.setdiff1d(np.arange(M), [M // 2, M - 1])
+    assert np.array_equal(z[other].view(np.uint32), plain[other].view(np.uint32))
+    assert np.isnan(z[M - 1]).all()
+    if M // 2 != M - 1:
+        w = W[K - 1]
+        assert np.array_equal(z[M // 2][w != 0], np.where(w > 0, np.inf, -np.inf)[w != 0].astype(np.float32))
+        assert np.isnan(z[M // 2][w == 0]).all()
 
 
 def test_gemm_split_counters_survive_other_workspace_users(dev, orc):
