@@ -23,6 +23,7 @@
 #include "conv_common.hpp"
 #include "mfma_core.hpp"
 #include "tbn_f4.hpp"
+#include "tbn_waves.hpp"
 
 namespace {
 
@@ -690,6 +691,16 @@ int tbn_hip_qlinear_matmul_binary_tbn(const float* A, int64_t lda, int64_t M, in
         if (hipMemset2DAsync(out, ldo * sizeof(float), 0, N * sizeof(float), M, s) != hipSuccess)
             return tbn_hip::fail(TBN_RUNTIME_ERROR, "hipMemset2DAsync failed");
         return tbn_hip::ok();
+    }
+    const int plan = tbn_hip::tbn_waves_plan(static_cast<int>(M), static_cast<int>(N));
+    // one launch where that is faster; shapes that the passes below refuse
+    // (8 GiB of operands, ldo of 2^21) stay with them
+    if (plan >= 0 && M * (K_pad / 8) + N_pad * (K_pad / 32) < (int64_t{1} << 31) && ldo < (1 << 21) &&
+        lda <= (1 << 22) && reinterpret_cast<uintptr_t>(packed) % 4 == 0) {
+        const tbn_hip::TbnWavesArgs a{A, lda, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), packed,
+                                      K_pad / 8, static_cast<int>(K_pad), static_cast<int>(N_pad), scale, lo, hi, out,
+                                      ldo};
+        return tbn_hip::tbn_waves(a, plan, s);
     }
     Scratch scr;
     scr.stream = s;

@@ -201,7 +201,7 @@ int tbn_hip_quantize_pack_ternary_f32(const float* w, int64_t K, int64_t N, int 
  * scale: per-column fp32 [N] or NULL (then s = 1); alpha: scalar multiplier
  * (the reference's scalar `scale` argument); bias: [N] or NULL.
  * C: fp32 [M, N], ldc >= N.  Requires K_pad % 32 == 0, K_pad >= K, N_pad >= N.
- * Shapes whose tiles would not fill the chip split K over blocks and keep the
+ * A K split over blocks, which only the tuning controls ask for, keeps its
  * partial sums in the library's per-device stream workspace; those calls
  * return TBN_NOT_IMPLEMENTED while the stream captures.
  * Replaces tbn::qlinear_matmul_binary / _blocked_packed / _naive
@@ -494,8 +494,10 @@ int tbn_hip_tbn_gemm_scaled(const uint8_t* pos, const uint8_t* neg, const uint8_
 /* qlinear_matmul_binary as the reference computes it (quantized_gemm_neon.cpp:
  * 160-243,380-430): out[M, N] = float(sum_k t(A[m,k]) * w[k,n]) * scale with
  * t the ternarization at (lo, hi) and w the packed BinaryMatrix (K_pad % 64
- * == 0, K_pad < 2^24, N_pad >= N).  Uses the stream workspace for the fp4
- * operand rows: M*K_pad/2 (rounded up to 256) + N_pad*K_pad/2 bytes. */
+ * == 0, K_pad < 2^24, N_pad >= N).  Products of at most 256 tiles of 32 x 256
+ * run in one launch; larger ones use the stream workspace for the fp4 operand
+ * rows: M*K_pad/2 (rounded up to 256) + N_pad*K_pad/2 bytes, and return
+ * TBN_NOT_IMPLEMENTED while the stream captures. */
 int tbn_hip_qlinear_matmul_binary_tbn(const float* A, int64_t lda, int64_t M, int64_t K,
                                       const uint8_t* packed, int64_t K_pad, int64_t N,
                                       int64_t N_pad, float scale, float lo, float hi, float* out,

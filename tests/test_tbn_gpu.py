@@ -206,6 +206,43 @@ def test_qlinear_tbn_leaves_memory_past_the_output_alone(dev, orc, M, N, ldo):
     assert np.array_equal(out[:, N:].view(np.uint32), guard[:, N:]), "columns past N were written"
 
 
+# every tile of the one-launch kernel, one past its last size, K around a
+# lane's 32 and a step's 64 / 128 values, padding beyond the next multiple of
+# 64, thresholds that ternarize the padding's zeros to -1 and +1, and rows that are not
+# 16-byte aligned
+@pytest.mark.parametrize("M,K,N,K_pad,lo,hi", [
+    (1, 1, 1, 64, -0.1, 0.1), (16, 129, 257, 192, -0.1, 0.1), (15, 2047, 4096, 2048, -0.25, 0.1),
+    (48, 320, 2001, 384, -0.1, 0.1), (63, 1000, 4090, 1088, 0.05, 0.3), (130, 63, 2000, 64, -0.1, 0.1),
+    (250, 577, 4000, 640, -0.3, -0.05), (1000, 65, 1030, 128, -0.1, 0.1), (1020, 257, 2048, 512, 0.2, -0.2),
+    (700, 130, 4000, 192, -0.1, 0.1)])
+def test_qlinear_tbn_one_launch_tiles(dev, M, K, N, K_pad, lo, hi):
+    """Bit for bit against the integer product in float64, and nothing written
+    outside the output."""
+    A = special_matrix(M, K, seed=M + K + N)
+    rng = np.random.default_rng(N)
+    N_pad = (N + 7) // 8 * 8
+    binw = (rng.random((K, N)) < 0.5).astype(np.uint8)
+    packed = empty(N_pad * K_pad // 8, torch.uint8)
+    tbn_hip.call("tbn_hip_pack_binary", P(to_dev(binw)), K, N, tbn_hip.LAYOUT_KN, K_pad, N_pad, P(packed), None)
+    lda, ldo = K + 3, N + 2
+    wide = np.full((M, lda), np.nan, np.float32)
+    wide[:, :K] = A
+    dA = to_dev(np.concatenate([np.float32([np.nan]), wide.reshape(-1)]))
+    out = torch.full(((M + 2) * ldo,), float("nan"), device=dev)
+    tbn_hip.call("tbn_hip_qlinear_matmul_binary_tbn", dA.data_ptr() + 4, lda, M, K, P(packed), K_pad, N, N_pad, 0.37,
+                 lo, hi, P(out), ldo, None)
+
+    def ternary(v):
+        return np.where(v < np.float32(lo), -1.0, np.where(v > np.float32(hi), 1.0, 0.0))
+
+    C = ternary(A) @ (binw * 2.0 - 1.0) + (K_pad - K) * ternary(np.zeros(1, np.float32))  # padding weights are +1
+    want = C.astype(np.float32) * np.float32(0.37)
+    full = host(out)
+    y = full[:M * ldo].reshape(M, ldo)
+    assert np.array_equal(y[:, :N].view(np.uint32), want.view(np.uint32))
+    assert np.isnan(y[:, N:]).all() and np.isnan(full[M * ldo:]).all(), "written outside the output"
+
+
 def test_qlinear_tbn_headline_shape_exact(dev):
     """4096^3: every element equals float(exact integer product) * scale
     (the integer product formed in float64 on the GPU, exact below 2^53)."""
