@@ -218,3 +218,60 @@ def test_avgpool2d_and_global_maxpool2d(dev, tbn, orc, on_device):
     assert np.array_equal(y, orc.avgpool2d(x, (3, 3), (2, 2), (1, 1), count_include_pad=True))
     g = _out(tbn.global_maxpool2d(a), on_device)
     assert np.array_equal(g.reshape(2, 8), orc.global_maxpool2d(x))
+
+
+def test_released_block_waits_for_its_stream(dev, tbn):
+    """A block released on a busy stream goes back to that stream at once, to
+    another thread's stream only when the first has run dry, and to any stream
+    after the thread that released it has moved on (which waits)."""
+    import threading
+
+    import torch
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    x = torch.randn((4096, 4096), device=dev)
+    shape = [1237, 1009]  # a size class of its own here
+    tbn.empty_cache()
+
+    def on_b():
+        got = []
+
+        def work():
+            tbn.set_current_stream(b.cuda_stream)
+            got.append(tbn.Tensor.empty(shape))
+            tbn.set_current_stream(0)
+
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        return got[0]
+
+    tbn.set_current_stream(a.cuda_stream)
+    try:
+        block = tbn.Tensor.empty(shape)
+        ptr = block.data_ptr()
+        del block
+        again = tbn.Tensor.empty(shape)
+        assert again.data_ptr() == ptr
+        with torch.cuda.stream(a):
+            for _ in range(200):
+                x = (x @ x) * 1e-3
+        del again  # released while its stream is busy
+        busy = not a.query()
+        other = on_b()
+        if busy:
+            assert other.data_ptr() != ptr
+        a.synchronize()
+        third = on_b()
+        assert third.data_ptr() == ptr
+        del other, third
+        block = tbn.Tensor.empty(shape)
+        ptr = block.data_ptr()
+        with torch.cuda.stream(a):
+            x = x @ x
+        del block
+    finally:
+        tbn.set_current_stream(0)  # waits for stream a
+    final = tbn.Tensor.empty(shape)
+    assert final.data_ptr() == ptr
+    tbn.empty_cache()
