@@ -105,6 +105,25 @@ def test_quantize_pack_binary_gemm_sampled(dev, orc, K, N, passes):
     assert np.array_equal(host(out), orc.pack_binary(binw, K, N, tbn_hip.LAYOUT_KN, K_pad, N_pad))
 
 
+# BINARY bytes [K, N] around a thread's 4 columns, a block's 128 columns, a
+# word's 32 and a block's 256 rows, with bytes that are neither 0 nor 1 and a
+# tensor that starts off a 4-byte boundary
+@pytest.mark.parametrize("K,N", [(1, 3), (1, 4), (31, 5), (32, 126), (33, 127), (257, 129), (300, 130), (255, 511), (64, 4099)])
+@pytest.mark.parametrize("extra", [0, 256], ids=["tight", "padded"])
+def test_pack_binary_bytes_tiles(dev, orc, K, N, extra):
+    rng = np.random.default_rng(K * N)
+    b = rng.choice(np.uint8([0, 1, 1, 2, 127, 128, 129, 255]), size=K * N + 1)
+    K_pad, N_pad = tbn_hip.padded_dims(K, N)
+    K_pad, N_pad = K_pad + extra, N_pad + (8 if extra else 0)
+    out = torch.full((N_pad * K_pad // 8 + 64,), 0x5A, dtype=torch.uint8, device=dev)
+    tbn_hip.call("tbn_hip_pack_binary", to_dev(b).data_ptr() + 1, K, N, tbn_hip.LAYOUT_KN, K_pad, N_pad, P(out), None)
+    full = host(out)
+    bits = np.zeros((N_pad, K_pad), np.uint8)  # padding is +1: bit 0
+    bits[:N, :K] = b[1:].reshape(K, N).T != 1
+    assert np.array_equal(full[:-64], np.packbits(bits, axis=1, bitorder="little").reshape(-1))
+    assert (full[-64:] == 0x5A).all()
+
+
 @pytest.mark.parametrize("n", [1, 4, 5, 1001, 4096 * 4096])
 def test_pack_ternary2_bit_exact(dev, orc, n):
     rng = np.random.default_rng(n)
