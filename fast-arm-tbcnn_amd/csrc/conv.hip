@@ -290,6 +290,8 @@ int tbn_hip_conv2d_f32(const float* x, const tbn_conv2d_desc* desc, const float*
     TBN_DEVICE_GUARD();
     if (tbn_hip::conv_stem_supported(desc, flags))
         return tbn_hip::conv_stem_run(x, desc, w, bias, flags, y, tbn_hip::stream_of(stream));
+    if (tbn_hip::conv_dense_supported(desc))
+        return tbn_hip::conv_dense_run(x, desc, w, bias, flags, y, tbn_hip::stream_of(stream));
     if (tbn_hip::conv_small_supported(desc))
         return tbn_hip::conv_small_run(0, x, desc, w, 0, nullptr, 1.0f, bias, nullptr, flags, y,
                                        tbn_hip::stream_of(stream));

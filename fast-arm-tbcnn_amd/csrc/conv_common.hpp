@@ -159,6 +159,11 @@ int64_t conv_patch_scratch_bytes(int weights, const tbn_conv2d_desc* desc, int f
 bool conv_stem_supported(const tbn_conv2d_desc* desc, int flags);
 int conv_stem_run(const float* x, const tbn_conv2d_desc* desc, const float* w, const float* bias, int flags,
                   float* y, hipStream_t s);
+// fp32 layers on the fp32 matrix instructions (conv_dense.hip), chosen from
+// one image's shape only.
+bool conv_dense_supported(const tbn_conv2d_desc* desc);
+int conv_dense_run(const float* x, const tbn_conv2d_desc* desc, const float* w, const float* bias, int flags,
+                   float* y, hipStream_t s);
 // Small layers (conv_small.hip): one image and a channel group per block,
 // staged in LDS, fp32 FMAs; chosen from one image's shape only.
 bool conv_small_supported(const tbn_conv2d_desc* desc);

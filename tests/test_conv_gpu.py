@@ -699,3 +699,51 @@ def test_conv_pair_declines_split_and_other_shapes(dev):
             tbn_hip.call("tbn_hip_conv2d_f32_prepacked_pair", tbn_hip.WEIGHTS_BINARY, None, d, None, None, 1.0, None,
                          None, 0, None, None, None, 1.0, None, 0, None, 2, None)
         assert e.value.code == tbn_hip.NOT_IMPLEMENTED
+
+
+# tiles of 64 x 64, 32 x 32 and 16 x 16 of the fp32 kernel with ragged
+# channels and positions, K around its chunks, windows that cross images inside a tile
+# (planes of 1 to 49 positions), stride, dilation, padding wider than the kernel's
+# reach, and the fused pool over odd planes
+@pytest.mark.parametrize("n,c,h,w,m,kh,kw,s,p,d", [
+    (40, 17, 19, 23, 70, 3, 3, 1, 1, 1), (9, 33, 28, 27, 65, 1, 1, 1, 0, 1), (30, 5, 31, 33, 20, 5, 5, 1, 2, 1),
+    (17, 40, 3, 3, 33, 3, 3, 1, 0, 1), (65, 64, 1, 1, 48, 1, 1, 1, 0, 1), (3, 13, 7, 7, 5, 5, 5, 1, 2, 1),
+    (2, 70, 9, 15, 130, 3, 3, 2, 1, 1), (5, 36, 12, 11, 24, 3, 2, 1, 2, 2), (1, 129, 5, 6, 17, 3, 3, 3, 4, 1),
+    (2, 9, 40, 9, 12, 1, 7, 1, 3, 1), (1, 3, 30, 30, 16, 5, 5, 2, 0, 3)])
+@pytest.mark.parametrize("flags", [0, tbn_hip.EPI_RELU, tbn_hip.EPI_RELU | tbn_hip.EPI_MAXPOOL2X2], ids=["plain", "relu", "pool"])
+def test_conv_f32_dense_tiles(dev, n, c, h, w, m, kh, kw, s, p, d, flags):
+    """fp32 conv against torch in float64 on the CPU, within the rounding of
+    K fp32 sums; the last image alone gives the same bits; nothing is written
+    past the output."""
+    rng = np.random.default_rng(n + c * 3 + m)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = rng.standard_normal((m, c, kh, kw)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+
+    def ref(xx, ww, bb):
+        return torch.nn.functional.conv2d(torch.from_numpy(xx).double(), torch.from_numpy(ww).double(),
+                                          torch.from_numpy(bb).double(), s, p, d)
+
+    want = ref(x, wt, b)
+    room = ref(np.abs(x), np.abs(wt), np.abs(b)) * ((c * kh * kw + 4) * 2.0 ** -24)
+    pool = bool(flags & tbn_hip.EPI_MAXPOOL2X2)
+    if pool and min(want.shape[2:]) < 2:
+        pytest.skip("no 2x2 window")
+    if flags & tbn_hip.EPI_RELU:
+        want = want.clamp_min(0)
+    if pool:
+        want, room = torch.nn.functional.max_pool2d(want, 2), torch.nn.functional.max_pool2d(room, 2)
+
+    def run(xx):
+        shape = (xx.shape[0],) + tuple(want.shape[1:])
+        size = int(np.prod(shape))
+        y = torch.full((size + 64,), float("nan"), device=dev)
+        desc = tbn_hip.conv_desc(xx.shape[0], c, h, w, m, kh, kw, s, s, p, p, d, d)
+        tbn_hip.call("tbn_hip_conv2d_f32", P(to_dev(xx)), desc, P(to_dev(wt)), P(to_dev(b)), flags, P(y), None)
+        full = host(y)
+        assert np.isnan(full[size:]).all(), "written past the output"
+        return full[:size].reshape(shape)
+
+    y = run(x)
+    assert (np.abs(y - want.numpy()) <= room.numpy()).all()
+    assert np.array_equal(run(x[-1:].copy()).view(np.uint32), y[-1:].view(np.uint32))
