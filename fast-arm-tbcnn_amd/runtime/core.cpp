@@ -195,13 +195,16 @@ void* allocate(size_t bytes) {
         };
         if (void* b = take()) return b;
         // only blocks of other streams are left: ask those streams, unless
-        // this thread's stream captures (a query could end the capture)
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        const bool capturing = hipStreamIsCapturing(static_cast<hipStream_t>(t_stream), &st) != hipSuccess ||
-                               st != hipStreamCaptureStatusNone;
-        if (!capturing) {
+        // this thread's stream or the one asked captures (a query could end the
+        // capture)
+        auto capturing = [](Stream s) {
+            hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+            return hipStreamIsCapturing(static_cast<hipStream_t>(s), &st) != hipSuccess ||
+                   st != hipStreamCaptureStatusNone;
+        };
+        if (!capturing(t_stream)) {
             for (size_t i = 0; i < v.size(); ++i) {
-                if (!v[i].pending) continue;
+                if (!v[i].pending || capturing(v[i].stream)) continue;
                 const hipError_t q = hipStreamQuery(static_cast<hipStream_t>(v[i].stream));
                 if (q == hipErrorNotReady) continue;
                 if (q == hipSuccess) settled_locked(p, dev, v[i].stream, p.releases);

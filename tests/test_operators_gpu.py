@@ -275,3 +275,58 @@ def test_released_block_waits_for_its_stream(dev, tbn):
     final = tbn.Tensor.empty(shape)
     assert final.data_ptr() == ptr
     tbn.empty_cache()
+
+
+def test_capturing_stream_is_not_asked_for_a_block(dev, tbn):
+    """A block that a stream released before its capture began leaves the
+    capture alone when another thread looks for a block of that size."""
+    import threading
+
+    import torch
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    x, y = torch.arange(64.0, device=dev), torch.zeros(64, device=dev)
+    shape = [1237, 1009]  # a size class of its own here
+    torch.add(x, 1, out=y)
+    torch.cuda.synchronize()
+    tbn.empty_cache()
+    ready, capturing, done = threading.Event(), threading.Event(), threading.Event()
+    got = []
+
+    def work():
+        tbn.set_current_stream(b.cuda_stream)
+        ready.set()
+        capturing.wait(30)
+        try:
+            got.append(tbn.Tensor.empty(shape))
+        finally:
+            done.set()
+
+    t = threading.Thread(target=work)
+    t.start()
+    assert ready.wait(30)
+    tbn.set_current_stream(a.cuda_stream)
+    try:
+        block = tbn.Tensor.empty(shape)
+        ptr = block.data_ptr()
+        del block
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.stream(a):
+            graph.capture_begin(capture_error_mode="thread_local")
+            torch.add(x, 2, out=y)
+            capturing.set()
+            done.wait(30)
+            graph.capture_end()
+        t.join()
+        assert got[0].data_ptr() != ptr
+        for _ in range(3):
+            y.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(a):
+                graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, x + 2)
+    finally:
+        capturing.set()
+        tbn.set_current_stream(0)
+        tbn.empty_cache()
